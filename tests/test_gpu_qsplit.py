@@ -82,6 +82,29 @@ def test_a_token_with_an_infinity_touches_no_other(ctx, dtype):
     assert not np.any(np.isfinite(got[[2, 4]]))
 
 
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_an_infinity_takes_the_signs_of_the_weights(ctx, dtype):
+    """inf * w: infinite by w's sign, NaN where w is 0 or two infinities meet
+    with opposite signs, as in the f32 sums of the vector form."""
+    rng = np.random.default_rng(10)
+    rows, cols, n = 1100, 512, 8
+    raw = blocks(dtype, rows, cols, rng)
+    x = rng.normal(size=(n, cols)).astype(np.float32)
+    x[1, 300] = np.inf
+    x[3, 511] = -np.inf
+    x[6, 0], x[6, 40] = np.inf, np.inf
+    got = streamed(ctx, QuantMatrix(ctx, dtype, rows, cols, raw), (x, n)).reshape(n, rows)
+    w = weights(dtype, raw, rows, cols)
+    for t, at in ((1, [300]), (3, [511]), (6, [0, 40])):
+        with np.errstate(invalid="ignore"):
+            want = sum(x[t, c].astype(np.float64) * w[:, c] for c in at)
+        # w = d sc q - dmin m rounds in f32: its sign is sure away from zero
+        ok = np.all([(np.abs(w[:, c]) > 1e-5 * np.abs(w).max(1)) | (w[:, c] == 0) for c in at], axis=0)
+        assert ok.sum() > rows // 2
+        assert np.array_equal(got[t][ok], want[ok].astype(np.float32), equal_nan=True), (t, at)
+        assert not np.any(np.isfinite(got[t]))
+
+
 def test_a_quantised_tail_past_the_matrix_is_not_used(ctx):
     """The last row's last span is read in 16-byte pieces that end with the
     matrix: bytes behind it (here NaN scales) must not reach the result."""
