@@ -763,6 +763,69 @@ __global__ __launch_bounds__(kThreads) void pf_heads_kernel(PfHeads a)
 constexpr int kAttnPos = 64; // positions per K/V tile
 constexpr int kVStride = 68; // halves per V^T row in LDS: 8-byte reads of 32 rows touch every bank once
 
+// One query row in f32 on one wavefront, as the decode step sums it.  For
+// workgroups whose tiles hold an inf or NaN (an f16 key or value that
+// overflowed): in the products above it reaches rows that do not attend it
+// (0 * inf) and a -inf score, which weighs 0, may become NaN (hi * inf + lo *
+// inf).  Lanes hold HD / 64 neighbouring dimensions.
+template <int HD>
+__device__ __forceinline__ void attn_row_f32(const PfAttn &a, const _Float16 *kc, const _Float16 *vc, int kvh, int client,
+                                             int t, int g, int lane)
+{
+    constexpr int EPL = HD / EMU_WAVE;
+    const int qpos = (int)a.positions[client] + t, lo = a.window > 0 && qpos + 1 > a.window ? qpos + 1 - a.window : 0;
+    const size_t tok = (size_t)client * a.tc + t;
+    const int head = kvh * (a.heads / a.kv_heads) + g, c = lane * EPL;
+    const _Float16 *qp = a.q + (tok * a.heads + head) * 2 * HD + c;
+    const float qs = a.q_scale[tok * a.heads + head];
+    float q[EPL], acc[EPL], m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+        q[e] = ((float)qp[e] + (float)qp[HD + e]) * qs;
+        acc[e] = 0.0f;
+    }
+    constexpr int NP = 8; // positions whose loads are in flight together
+#pragma unroll 1
+    for (int p0 = lo; p0 <= qpos; p0 += NP) {
+        float k[NP][EPL], v[NP][EPL], s[NP], mn = m;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const size_t at = (size_t)(p0 + i <= qpos ? p0 + i : qpos) * HD + c;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+                k[i][e] = (float)kc[at + e];
+                v[i][e] = (float)vc[at + e];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            float d = 0.0f;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) d = __builtin_fmaf(q[e], k[i][e], d);
+            d = wave_sum(d);
+            d = a.score_div > 0.0f ? d / a.score_div : d * a.score_mul;
+            s[i] = p0 + i <= qpos ? d : -INFINITY;
+            mn = fmaxf(mn, s[i]);
+        }
+        const float f = m == -INFINITY ? 0.0f : expf(m - mn);
+        m = mn;
+        l *= f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[e] *= f;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const bool in = p0 + i <= qpos;
+            const float w = s[i] == -INFINITY ? 0.0f : expf(s[i] - m);
+            l += w;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[e] = in ? __builtin_fmaf(w, v[i][e], acc[e]) : acc[e];
+        }
+    }
+    float *out = a.out + tok * (size_t)(a.heads * HD) + (size_t)head * HD + c;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) out[e] = acc[e] / l;
+}
+
 template <int HD, int WV>
 __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel(PfAttn a)
 {
@@ -773,7 +836,7 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
     __shared__ __align__(16) _Float16 vt[HD * kVStride];
     constexpr bool kLoLds = HD > 64; // the queries' lo halves in LDS, not registers
     __shared__ __align__(16) _Float16 q_lo[kLoLds ? WV : 1][kLoLds ? NS * 64 * 8 : 8];
-    __shared__ uint64_t bad_s; // positions of the tile whose V row holds an inf or NaN
+    __shared__ int bad_s; // a key or value of the tiles is an inf or NaN
     const int tid = threadIdx.x, lane = tid & (EMU_WAVE - 1), w = tid / EMU_WAVE;
     const int kh = lane >> 5, j32 = lane & 31;
     const int kvh = blockIdx.y, client = blockIdx.z, G = a.heads / a.kv_heads;
@@ -818,7 +881,7 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[d][i] = 0.0f;
     float m = -INFINITY, l = 0.0f;
-    bool poison = false;
+    if (tid == 0) bad_s = 0;
 
     uint4 kr[KP], va[VP], vb[VP];
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
@@ -846,23 +909,18 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
     fetch(start);
     for (int p0 = start; p0 < end; p0 += kAttnPos) {
         __syncthreads();
-        if (tid == 0) bad_s = 0;
-        __syncthreads();
+        bool bad = false;
 #pragma unroll
         for (int i = 0; i < KP; ++i) { // operand order: position tile, 16-dim slice, lane
             const int x = tid + i * NT, p = x / (HD / 8), g = x % (HD / 8);
             *reinterpret_cast<uint4 *>(ks + ((size_t)((p >> 5) * NS + (g >> 1)) * 64 + (g & 1) * 32 + (p & 31)) * 8) = kr[i];
+            bad |= any_bad(kr[i]);
         }
 #pragma unroll
         for (int i = 0; i < VP; ++i) {
             const int x = tid + i * NT, gl = x & 7, p = ((x >> 3) & 7) + 8 * ((x / 64) % 4), g = 8 * (x / 256) + gl;
-            uint4 u = va[i], v = vb[i];
-            const bool bu = any_bad(u), bv = any_bad(v);
-            if (bu || bv) { // rare: keep them out of the product, mark the positions
-                if (bu) u = zero;
-                if (bv) v = zero;
-                atomicOr((unsigned long long *)&bad_s, (bu ? 1ull << (2 * p) : 0ull) | (bv ? 2ull << (2 * p) : 0ull));
-            }
+            const uint4 u = va[i], v = vb[i];
+            bad |= any_bad(u) || any_bad(v);
             const uint32_t lo[4] = {u.x, u.y, u.z, u.w}, hi[4] = {v.x, v.y, v.z, v.w};
             uint32_t *dst = reinterpret_cast<uint32_t *>(vt) + (size_t)(8 * g) * (kVStride / 2) + p;
 #pragma unroll
@@ -871,6 +929,7 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
                 dst[(2 * e + 1) * (kVStride / 2)] = (lo[e] >> 16) | (hi[e] & 0xffff0000u);
             }
         }
+        if (bad) bad_s = 1;
         __syncthreads();
         if (p0 + kAttnPos < end) fetch(p0 + kAttnPos);
         if (!w_live || p0 > w_last) continue; // uniform per wavefront; the barriers above are not skipped
@@ -889,7 +948,6 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
                     sc[pt] = mfma(kf, ql[s], sc[pt]);
             }
         }
-        const uint64_t bad = bad_s;
         const bool edge = p0 + kAttnPos - 1 > w_first || p0 < w_lo; // uniform per wavefront: some are masked
         float mx = -INFINITY;
 #pragma unroll
@@ -902,15 +960,6 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
                 // a NaN score reaches the row's sum through exp2 below
                 mx = fmaxf(mx, sc[pt][i]);
             }
-        if (bad) { // uniform over the workgroup
-#pragma unroll
-            for (int pt = 0; pt < 2; ++pt)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int q = 32 * pt + 8 * (i >> 2) + 4 * kh + (i & 3);
-                    if ((bad >> q & 1) && p0 + q <= qpos && p0 + q >= qlo) poison = true;
-                }
-        }
         mx = fmaxf(mx, emu_xor_get<32>(mx));
         const float mn = fmaxf(m, mx);
         const float ms = (mn == -INFINITY ? 0.0f : mn) - 15.0f; // nothing attended yet: all weights 0
@@ -946,11 +995,14 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
             }
         }
     }
+    if (bad_s) { // uniform over the workgroup; the last tile's barrier stands behind the last write
+        for (int i = r0 + 32 * w; i < min(r0 + 32 * (w + 1), rows); ++i)
+            attn_row_f32<HD>(a, kc, vc, kvh, client, i / G, i % G, lane);
+        return;
+    }
     l += emu_xor_get<32>(l);
-    const float other = emu_xor_get<32>(poison ? 1.0f : 0.0f);
     if (rq >= rows) return;
-    float inv = 1.0f / l;
-    if (poison || other != 0.0f) inv = __int_as_float(0x7fc00000);
+    const float inv = 1.0f / l;
     float *out = a.out + tok * (size_t)(a.heads * HD) + (size_t)head * HD + 4 * kh;
 #pragma unroll
     for (int d = 0; d < ND; ++d)

@@ -13,7 +13,7 @@ from dataclasses import replace
 import numpy as np
 import pytest
 
-from emufpga_amd import _lib
+from emufpga_amd import _lib, gguf
 from emufpga_amd.serve import QWEN3_8B_Q6K, Model, Session
 from tests.test_gpu_model import SMALL_QWEN3, SMALL_SMOL
 from tests.test_gpu_moe_model import gemma_layer_scales, small_gemma, small_granite, small_olmoe
@@ -120,3 +120,64 @@ def test_weights_written_after_a_prompt_are_the_ones_used(ctx):
     step_by_step(b, prompts)
     x, y = a.read_kv(0, 0, True, 40), b.read_kv(0, 0, True, 40)
     assert np.all(np.isfinite(y)) and np.linalg.norm(x - y) <= 2.0 ** -10 * np.linalg.norm(y)
+
+
+D_AT = {_lib.Q6_K: [208], _lib.Q5_K: [0, 2], _lib.Q2_K: [80, 82], _lib.Q8_0: [0]}  # a block's f16 factors
+
+
+def scale_rows(model, first, rows, factor):
+    """Rows first .. first + rows - 1 of layer 0's q, k, v times `factor`."""
+    enc = model.cfg.encoding
+    be, bb = gguf.LAYOUT[enc]
+    blob = model.read_tensor(_lib.EMU_T_LAYER, 0)
+    rb = model.cfg.hidden // be * bb
+    part = blob[first * rb:(first + rows) * rb].reshape(-1, bb)
+    for at in D_AT[enc]:
+        d = (part[:, at:at + 2].copy().view(np.float16).astype(np.float64) * factor).astype(np.float16)
+        assert np.all(np.isfinite(d))
+        part[:, at:at + 2] = d.view(np.uint8)
+    model.write_tensor(_lib.EMU_T_LAYER, blob, 0)
+
+
+@pytest.mark.parametrize("what", ["keys", "values"])
+@pytest.mark.parametrize("form", ["q6_k", "q5_k_no_groups", "q2_k_head256"])
+def test_cache_entries_that_overflow_f16(ctx, form, what):
+    """A key or value past f16's range is infinite in the cache.  A query whose
+    score with such a key is -inf passes over it; where the steps give a
+    finite row the pass does, and the same one, and nowhere else."""
+    cfg = replace(FORMS[form], layers=2, heads=FORMS[form].kv_heads)
+    model = Model(ctx, cfg)
+    model.synth(3)
+    n, plen, hd = 2, 150, cfg.head_dim
+    prompts = np.random.default_rng(8).integers(0, cfg.vocab, size=(n, plen)).astype(np.uint32)
+    a, b = (Session(model, n, plen + 2) for _ in range(2))
+    if what == "keys":  # one normalised dimension of layer 0's keys, small in its queries
+        q_gain, k_gain = (np.ones((cfg.layers, hd), np.float32) for _ in range(2))
+        k_gain[0, 5] = 65504 / (1.6 if cfg.kv_heads == 1 else 2.3)
+        q_gain[0, [5, 5 + hd // 2]] = 1e-5
+        model.write_tensor(_lib.EMU_T_K_NORM, k_gain)
+        model.write_tensor(_lib.EMU_T_Q_NORM, q_gain)
+    else:  # one value row, past the range for its largest token alone
+        step_by_step(b, prompts)
+        v = b.read_kv(0, 0, True, plen)[:, 3]
+        b.reset()
+        top = int(np.argmax(np.abs(v)))
+        prompts[0, [top, 80]] = prompts[0, [80, top]]
+        scale_rows(model, cfg.q_width + cfg.kv_width + 3, 1, 65504 * 1.02 / np.abs(v).max())
+    a.generate(prompts, 1)
+    step_by_step(b, prompts)
+    after = 0  # rows of layer 1 that stay finite behind layer 0's first infinity
+    for c in range(n):
+        first = plen
+        for layer in range(2):
+            for values in (False, True):
+                x, y = (s.read_kv(c, layer, values, plen) for s in (a, b))
+                assert np.array_equal(np.isfinite(x), np.isfinite(y)), (layer, values, c)
+                fine = np.all(np.isfinite(y), axis=1)
+                assert np.linalg.norm(x[fine] - y[fine]) <= 2.0 ** -10 * np.linalg.norm(y[fine])
+                if layer == 0 and values == (what == "values"):
+                    first = plen if fine.all() else int(np.argmin(fine))
+                if layer == 1 and first < plen:
+                    after += int(np.sum(fine[first:]))
+        assert first > 0 and (c or first < plen)
+    assert (after > 0) == (what == "keys")
