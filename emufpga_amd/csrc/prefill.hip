@@ -643,8 +643,8 @@ __global__ __launch_bounds__(kRowThreads) void pf_glu_kernel(const float *part, 
 
 // ---- heads: QK-norm, RoPE, KV append --------------------------------------
 // One wavefront per (token, head of q|k|v): queries go out as hi and lo
-// halves under one power of two per (token, head), keys and values rounded
-// to the cache's type (the arithmetic of attn_decode_kernel's preparation).
+// halves under one power of two per (token, head), or in f32 where the cache
+// holds f32 values, keys and values rounded to the cache's type (the arithmetic of attn_decode_kernel's preparation).
 __device__ __forceinline__ void kv_store(void *cache, int kv_f16, size_t at, float v)
 {
     if (kv_f16) static_cast<__half *>(cache)[at] = __float2half_rn(v);
@@ -730,11 +730,21 @@ __global__ __launch_bounds__(kThreads) void pf_heads_kernel(PfHeads a)
             }
         return;
     }
+    _Float16 *q = a.q + ((size_t)r * a.heads + item) * 2 * HD;
+    if (!a.kv_f16) { // an f32 cache is attended in f32: the queries as they are, in the same bytes
+        float *q32 = reinterpret_cast<float *>(q);
+#pragma unroll
+        for (int j = 0; j < PPL; ++j)
+            if (lane + EMU_WAVE * j < NP) {
+                q32[ia[j]] = x[j];
+                q32[ib[j]] = y[j];
+            }
+        return;
+    }
     amax = emu_wave_reduce(amax, [](float p, float q) { return fmaxf(p, q); });
     const bool finite = amax <= 3.402823466e38f;
     float s, inv;
     pow2_scale(amax, s, inv);
-    _Float16 *q = a.q + ((size_t)r * a.heads + item) * 2 * HD;
 #pragma unroll
     for (int j = 0; j < PPL; ++j)
         if (lane + EMU_WAVE * j < NP) {
@@ -1041,10 +1051,9 @@ __global__ __launch_bounds__(kThreads) void pf_attn_f32_kernel(PfAttn a, int hd,
 #pragma unroll
     for (int g = 0; g < GH; ++g) {
         const int head = h0 + (g < nh ? g : 0);
-        const _Float16 *q = a.q + (tok * a.heads + head) * 2 * hd + piece * V;
-        const float s = a.q_scale[tok * a.heads + head];
+        const float *q = reinterpret_cast<const float *>(a.q) + (tok * a.heads + head) * hd + piece * V;
 #pragma unroll
-        for (int e = 0; e < V; ++e) qr[g][e] = ((float)q[e] + (float)q[hd + e]) * s; // 24 bits: one rounding
+        for (int e = 0; e < V; ++e) qr[g][e] = q[e];
     }
     float m[GH], l[GH], acc[GH][V];
 #pragma unroll

@@ -69,8 +69,8 @@ struct PfHeads {
     int rope_fma, interleaved, heads, kv_heads, layers, layer, context, tc;
     void *k_cache, *v_cache; // f16 or f32
     int kv_f16;
-    _Float16 *q;    // [row][head][hi, lo][head dim]
-    float *q_scale; // [row][head]
+    _Float16 *q;    // [row][head][hi, lo][head dim], or f32 [row][head][head dim] for an f32 cache
+    float *q_scale; // [row][head] (f16 cache)
 };
 int emu_pf_heads(emu_ctx *ctx, const PfHeads &a, int hd, int n);
 

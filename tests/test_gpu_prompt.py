@@ -84,6 +84,29 @@ def test_prompt_pass_over_an_f32_cache(ctx, form):
     compare(model, a, b, n, plen, rng.integers(0, model.cfg.vocab, size=n))
 
 
+@pytest.mark.parametrize("form", ["q5_k_no_groups", "q2_k_head256"])
+def test_queries_over_an_f32_cache_are_f32(ctx, form):
+    """Two query dimensions 2^24 times the others, over keys that hold zeros
+    there: the scores come from the others alone, and need all their bits.
+    Layer 1's entries carry layer 0's products' rounding (7e-7 of them; a pair
+    of halves under the head's largest would leave 6e-5)."""
+    model = Model(ctx, FORMS[form])
+    model.synth(12)
+    hd, layers = model.cfg.head_dim, model.cfg.layers
+    q_gain, k_gain = (np.ones((layers, hd), np.float32) for _ in range(2))
+    q_gain[:, [5, 5 + hd // 2]] = 2.0 ** 24
+    k_gain[:, [5, 5 + hd // 2]] = 0.0
+    model.write_tensor(_lib.EMU_T_Q_NORM, q_gain)
+    model.write_tensor(_lib.EMU_T_K_NORM, k_gain)
+    prompts = np.random.default_rng(7).integers(0, model.cfg.vocab, size=(2, 75)).astype(np.uint32)
+    a, b = (Session(model, 2, 77, kv_f16=False) for _ in range(2))
+    a.generate(prompts, 1)
+    step_by_step(b, prompts)
+    for layer in range(layers):
+        x, y = (s.read_kv(1, layer, True, 75) for s in (a, b))
+        assert np.linalg.norm(x - y) <= 3e-6 * np.linalg.norm(y), layer
+
+
 def test_prompts_longer_than_a_pass_after_a_replaced_client(ctx):
     """Eight clients of 300 tokens (two passes), one of them fresh while the
     others sit at position 40."""
