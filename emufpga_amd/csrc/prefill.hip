@@ -397,8 +397,13 @@ __device__ __forceinline__ void pf_tile(const PfGemm &g, uint8_t *lds, int a0, i
             }
         }
     };
-    // A span's sums start from zero and are added to the total at its end: one
-    // chain over 4096 columns (768 additions) rounds twice as far off.
+    // A stage's sums start from zero and are added to the total at its end.
+    // Against 64 bits the values' projection is off by 1.36e-7 of its norm at
+    // 576 columns and 1.5e-7 at 4096 so, by 1.94e-7 and 2.1e-7 with one addition
+    // per 256-column span, and by more than twice that in one chain.  (The
+    // small halves' products of a stage first, its hi * hi last: 1.1e-7 and
+    // 1.3e-7, but the operands spill at four fragments: 512 tokens of Qwen3-8B
+    // 28.1 -> 35.1 ms; the additions per stage cost 0.2.)
     float16v sum[L], acc[L];
 #pragma unroll
     for (int m = 0; m < L; ++m)
@@ -412,10 +417,6 @@ __device__ __forceinline__ void pf_tile(const PfGemm &g, uint8_t *lds, int a0, i
     }
     int buf = 0;
     for (int grp = s0 / PER; grp * PER < s1; ++grp) { // s0 is a multiple of PER
-#pragma unroll
-        for (int m = 0; m < L; ++m)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
             const int st = grp * PER + q;
@@ -431,6 +432,10 @@ __device__ __forceinline__ void pf_tile(const PfGemm &g, uint8_t *lds, int a0, i
             }
             if (q == 0) D::settle(cur);
             const uint8_t *ab = lds + buf * kBuf + (q % SB) * kFrags * 1024 + lane * 16;
+#pragma unroll
+            for (int m = 0; m < L; ++m)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 half8 bh, bl;
@@ -448,12 +453,12 @@ __device__ __forceinline__ void pf_tile(const PfGemm &g, uint8_t *lds, int a0, i
 #pragma unroll
                 for (int m = 0; m < L; ++m) acc[m] = mfma(ah[m], bl, acc[m]);
             }
+#pragma unroll
+            for (int m = 0; m < L; ++m)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sum[m][i] += acc[m][i];
             if (q % SB == SB - 1) buf ^= 1;
         }
-#pragma unroll
-        for (int m = 0; m < L; ++m)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) sum[m][i] += acc[m][i];
         cur = nxt;
     }
     if (row >= g.rows) return;

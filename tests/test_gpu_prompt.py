@@ -15,6 +15,7 @@ import pytest
 
 from emufpga_amd import _lib, gguf
 from emufpga_amd.serve import QWEN3_8B_Q6K, Model, Session
+from tests import npref
 from tests.test_gpu_model import SMALL_QWEN3, SMALL_SMOL
 from tests.test_gpu_moe_model import gemma_layer_scales, small_gemma, small_granite, small_olmoe
 
@@ -82,6 +83,30 @@ def test_prompt_pass_over_an_f32_cache(ctx, form):
         x, y = (s.read_kv(1, 0, values, plen) for s in (a, b))
         assert np.linalg.norm(x - y) <= 1e-5 * np.linalg.norm(y)
     compare(model, a, b, n, plen, rng.integers(0, model.cfg.vocab, size=n))
+
+
+@pytest.mark.parametrize("form", ["q6_k", "q5_k_no_groups", "q2_k_head256", "q8_0_smol", "q8_0_half_stage"])
+def test_products_against_64_bits(ctx, form):
+    """Layer 0's values over an f32 cache are the v rows' product with the
+    normalised embeddings, unrounded.  Bar: 1.7e-7 of the norm.  The halves
+    leave about 6e-8; a 64-column stage's sum takes 12 matrix instructions of
+    two roundings each (2.4e-8 sqrt(12) = 8e-8), and the 4 to 9 stages' sums
+    5e-8: 1.1e-7 to 1.4e-7 together.  256 columns in one chain leave 1.9e-7."""
+    cfg = FORMS[form]
+    model = Model(ctx, cfg)
+    model.synth(12)
+    prompts = np.random.default_rng(7).integers(0, cfg.vocab, size=(2, 75)).astype(np.uint32)
+    a = Session(model, 2, 77, kv_f16=False)
+    a.generate(prompts, 1)
+    rb = gguf.row_bytes(cfg.encoding, cfg.hidden)
+    blob = model.read_tensor(_lib.EMU_T_LAYER, 0)[(cfg.q_width + cfg.kv_width) * rb:][:cfg.kv_width * rb]
+    w, embed = (npref.DECODERS[cfg.encoding](raw).reshape(-1, cfg.hidden).astype(np.float64)
+                for raw in (blob, model.read_tensor(_lib.EMU_T_EMBED)))
+    for c in range(2):
+        x = embed[prompts[c, :74]]  # the last token is a decode step
+        want = x / np.sqrt((x * x).mean(1, keepdims=True) + cfg.eps) @ w.T
+        got = a.read_kv(c, 0, True, 74).astype(np.float64)
+        assert np.linalg.norm(got - want) <= 1.7e-7 * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("form", ["q5_k_no_groups", "q2_k_head256"])
