@@ -109,6 +109,35 @@ def test_products_against_64_bits(ctx, form):
         assert np.linalg.norm(got - want) <= 1.7e-7 * np.linalg.norm(want)
 
 
+def test_products_of_a_row_with_one_large_value(ctx):
+    """A normalised row with one column 2^20 times the others over zero
+    weights.  The others keep what test_products_against_64_bits holds, down to
+    2^-25 under the power of two that puts the largest into [2^14, 2^15): 2^-39
+    of it in each, times the weights' norm."""
+    cfg = FORMS["q8_0_smol"]
+    model = Model(ctx, cfg)
+    model.synth(12)
+    rb = gguf.row_bytes(cfg.encoding, cfg.hidden)
+    at = (cfg.q_width + cfg.kv_width) * rb
+    layer = model.read_tensor(_lib.EMU_T_LAYER, 0)
+    layer[at:at + cfg.kv_width * rb].reshape(cfg.kv_width, -1, 34)[:, 100 // 32, 2 + 100 % 32] = 0
+    model.write_tensor(_lib.EMU_T_LAYER, layer, 0)
+    gain = np.ones((cfg.layers, cfg.hidden), np.float32)
+    gain[0, 100] = 2.0 ** 20
+    model.write_tensor(_lib.EMU_T_ATTN_NORM, gain)
+    prompts = np.random.default_rng(7).integers(0, cfg.vocab, size=(1, 75)).astype(np.uint32)
+    a = Session(model, 1, 77, kv_f16=False)
+    a.generate(prompts, 1)
+    w = npref.DECODERS[cfg.encoding](layer[at:at + cfg.kv_width * rb]).reshape(-1, cfg.hidden).astype(np.float64)
+    embed = npref.DECODERS[cfg.encoding](model.read_tensor(_lib.EMU_T_EMBED)).reshape(-1, cfg.hidden).astype(np.float64)
+    x = embed[prompts[0, :74]]
+    x = x / np.sqrt((x * x).mean(1, keepdims=True) + cfg.eps) * gain[0]
+    want, got = x @ w.T, a.read_kv(0, 0, True, 74).astype(np.float64)
+    for t in range(74):
+        bar = 1.7e-7 * np.linalg.norm(want[t]) + 2.0 ** -39 * np.abs(x[t]).max() * np.linalg.norm(w)
+        assert np.linalg.norm(got[t] - want[t]) <= bar, t
+
+
 @pytest.mark.parametrize("form", ["q5_k_no_groups", "q2_k_head256"])
 def test_queries_over_an_f32_cache_are_f32(ctx, form):
     """Two query dimensions 2^24 times the others, over keys that hold zeros

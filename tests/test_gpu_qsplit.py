@@ -105,6 +105,30 @@ def test_an_infinity_takes_the_signs_of_the_weights(ctx, dtype):
         assert not np.any(np.isfinite(got[t]))
 
 
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_a_column_far_above_the_others(ctx, dtype):
+    """Activations 2^24 times the others over zero weights: the result comes
+    from the others, which keep 23 bits (a low half under the span's largest
+    value alone would leave them 2e-5).  Bar 3e-7 of the norm: the forms' sums
+    are off by 1.0e-7 to 2.6e-7 of it."""
+    rng = np.random.default_rng(12)
+    rows, cols, n = 4096, 4096, 8
+    raw = blocks(dtype, rows, cols, rng)
+    per = raw.reshape(rows, -1, npref.BLOCK_BYTES[dtype])
+    if dtype == _lib.Q8_0:
+        per[:, 100 // 32, 2 + 100 % 32] = 0
+    elif dtype == _lib.Q5_K:  # scale and minimum of columns 96..127
+        per[:, 0, [7, 11]] &= 0xC0
+    else:  # of columns 96..111
+        per[:, 0, 6] = 0
+    x = rng.normal(size=(n, cols)).astype(np.float32)
+    x[:, 100] = 3 * 2.0 ** 24
+    got = streamed(ctx, QuantMatrix(ctx, dtype, rows, cols, raw), (x, n)).reshape(n, rows)
+    want = x.astype(np.float64) @ weights(dtype, raw, rows, cols).T
+    for t in range(n):
+        assert np.linalg.norm(got[t] - want[t]) <= 3e-7 * np.linalg.norm(want[t]), t
+
+
 def test_a_quantised_tail_past_the_matrix_is_not_used(ctx):
     """The last row's last span is read in 16-byte pieces that end with the
     matrix: bytes behind it (here NaN scales) must not reach the result."""
