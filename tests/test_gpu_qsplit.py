@@ -30,7 +30,10 @@ def blocks(dtype, rows, cols, rng):
 @pytest.mark.parametrize("dtype,rows,cols", [
     (_lib.Q8_0, 1, 32), (_lib.Q8_0, 17, 288), (_lib.Q8_0, 40, 480), (_lib.Q8_0, 33, 2336), (_lib.Q5_K, 16, 256),
     (_lib.Q5_K, 31, 2304), (_lib.Q2_K, 1, 256), (_lib.Q2_K, 50, 2560), (_lib.Q8_0, 8193, 1024), (_lib.Q5_K, 8208, 1024),
-    (_lib.Q2_K, 8200, 1280)])
+    (_lib.Q2_K, 8200, 1280),
+    # the matrix-core form from two, three, five or six tokens on
+    (_lib.Q8_0, 4097, 64), (_lib.Q8_0, 16385, 32), (_lib.Q8_0, 2570, 2080), (_lib.Q8_0, 1031, 2336), (_lib.Q5_K, 2050, 512),
+    (_lib.Q5_K, 2065, 2304), (_lib.Q2_K, 16390, 256), (_lib.Q2_K, 2561, 2560)])
 def test_matvec_within_the_bar(ctx, dtype, rows, cols, n_tok):
     rng = np.random.default_rng(rows + cols + n_tok)
     raw = blocks(dtype, rows, cols, rng)
@@ -44,7 +47,7 @@ def test_matvec_within_the_bar(ctx, dtype, rows, cols, n_tok):
 
 @pytest.mark.parametrize("gain", [False, True])
 @pytest.mark.parametrize("n_tok", [3, 8])
-@pytest.mark.parametrize("dtype,rows,cols", [(_lib.Q8_0, 100, 544), (_lib.Q5_K, 1100, 1024), (_lib.Q2_K, 70, 768)])
+@pytest.mark.parametrize("dtype,rows,cols", [(_lib.Q8_0, 100, 544), (_lib.Q8_0, 1111, 544), (_lib.Q5_K, 1100, 1024), (_lib.Q2_K, 70, 768)])
 def test_gate_up_pair_within_the_bar(ctx, dtype, rows, cols, n_tok, gain):
     rng = np.random.default_rng(rows * 3 + n_tok)
     raws = [blocks(dtype, rows, cols, rng) for _ in range(2)]
