@@ -779,6 +779,7 @@ struct QmvArgs {
     int f32_act;           // f32 activations: the dequant + f32 FMA kernels, not the int8-limb ones
     int span_scales;       // multi-token chain: the A operands carry one scale per 256-column span
     int span_norm;         // with span_scales: apply the deferring link's RMS factor (with eps)
+    int lockstep;          // a session's step: at 2..8 tokens the form depends on the matrix, not on n_tok
 };
 
 // A matvec result's epilogue: divided by out_div (when set), then added to

@@ -1117,6 +1117,7 @@ int run_moe(emu_session *s)
         a.eps = c.eps;
         a.y = s->qkv;
         a.f32_act = s->f32();
+        a.lockstep = 1;
         if ((st = emu_launch_qmv(ctx, c.encoding, a, n)) != EMU_OK) return st;
         if ((st = emu_launch_attn(ctx, layer_attn(s, layer))) != EMU_OK) return st;
         QmvArgs o{};
@@ -1130,6 +1131,7 @@ int run_moe(emu_session *s)
         o.y = s->state;
         o.accumulate = 1;
         o.acc_scale = c.residual_scale;
+        o.lockstep = 1;
         if ((st = emu_launch_qmv(ctx, c.encoding, o, n)) != EMU_OK) return st;
         }
         emu_moe_desc d{};
@@ -1228,6 +1230,7 @@ int run_moe(emu_session *s)
                 ga.eps = c.eps;
                 g.y = s->act;
                 g.act = EMU_ACT_GELU_TANH;
+                g.lockstep = 1;
                 if ((st = emu_launch_qmv(ctx, c.encoding, g, n)) != EMU_OK) return st;
                 QmvArgs d{};
                 d.w = lw + m->off_sd;
@@ -1239,6 +1242,7 @@ int run_moe(emu_session *s)
                 d.y = s->state;
                 d.accumulate = 1;
                 d.acc_scale = c.residual_scale;
+                d.lockstep = 1;
                 if ((st = emu_launch_qmv(ctx, c.encoding, d, n)) != EMU_OK) return st;
             }
         } else {
@@ -1288,6 +1292,7 @@ int run_moe(emu_session *s)
     int slots = 0;
     // chained: the output on the matrix cores at any client count, as the
     // projections before it (a client's logits do not depend on the batch)
+    out.lockstep = 1;
     if ((st = chain ? emu_launch_mfma(ctx, c.encoding, out, n, &slots) : emu_launch_qmv(ctx, c.encoding, out, n, &slots)) !=
         EMU_OK)
         return st;
@@ -1332,6 +1337,7 @@ int run_step(emu_session *s)
         a.gain = reinterpret_cast<const float *>(m->base + m->off_attn_norm) + (size_t)layer * H;
         a.eps = c.eps;
         a.y = s->qkv;
+        a.lockstep = 1;
         if ((st = emu_launch_qmv(ctx, c.encoding, a, n)) != EMU_OK) return st;
         if ((st = emu_launch_attn(ctx, layer_attn(s, layer))) != EMU_OK) return st;
         // o projection + residual.
@@ -1345,6 +1351,7 @@ int run_step(emu_session *s)
         o.x = s->attn;
         o.y = s->state;
         o.accumulate = 1;
+        o.lockstep = 1;
         if ((st = emu_launch_qmv(ctx, c.encoding, o, n)) != EMU_OK) return st;
         // gate|up with the FFN RMSNorm and SwiGLU fused.
         QmvArgs g{};
@@ -1359,6 +1366,7 @@ int run_step(emu_session *s)
         g.gain = reinterpret_cast<const float *>(m->base + m->off_ffn_norm) + (size_t)layer * H;
         g.eps = c.eps;
         g.y = s->act;
+        g.lockstep = 1;
         if ((st = emu_launch_qmv(ctx, c.encoding, g, n)) != EMU_OK) return st;
         // down projection + residual.
         QmvArgs d{};
@@ -1371,6 +1379,7 @@ int run_step(emu_session *s)
         d.x = s->act;
         d.y = s->state;
         d.accumulate = 1;
+        d.lockstep = 1;
         if ((st = emu_launch_qmv(ctx, c.encoding, d, n)) != EMU_OK) return st;
         if ((st = mark(s, layer + 1)) != EMU_OK) return st;
     }
@@ -1393,6 +1402,7 @@ int run_step(emu_session *s)
     out.key_stride = (int)s->key_stride;
     out.tie_last = smol ? 1 : 0;
     int slots = 0;
+    out.lockstep = 1;
     if ((st = emu_launch_qmv(ctx, c.encoding, out, n, &slots)) != EMU_OK) return st;
     if ((st = launch_finalize(s, slots)) != EMU_OK) return st;
     return mark(s, c.layers + 1);

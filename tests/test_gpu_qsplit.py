@@ -5,13 +5,17 @@ test_qmatvec_random_within_tolerance (an f32 sum in another order).  Sizes: a
 row and a half tile, one span and less (32 columns), a last span of one block,
 eight wavefronts' spans and one more, two tiles per workgroup, and the sizes on
 both sides of the dispatch rule."""
+from dataclasses import replace
+
 import numpy as np
 import pytest
 
 import oracle
 from emufpga_amd import _lib
 from emufpga_amd.linear import QuantMatrix, streamed
+from emufpga_amd.serve import Model, Session
 from tests import npref
+from tests.test_gpu_model import SMALL_QWEN3, SMALL_SMOL
 
 pytestmark = pytest.mark.gpu
 
@@ -146,3 +150,37 @@ def test_a_quantised_tail_past_the_matrix_is_not_used(ctx):
     w = weights(_lib.Q8_0, raw, rows, cols)
     bound = 1e-5 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 1e-30
     assert np.all(np.abs(by.read(np.float32).reshape(n, rows) - ref.reshape(n, rows)) <= bound)
+
+
+@pytest.mark.parametrize("form", [
+    replace(SMALL_SMOL, vocab=4096), replace(SMALL_QWEN3, encoding=_lib.Q5_K, ffn=1280, vocab=3000),
+    replace(SMALL_QWEN3, encoding=_lib.Q2_K, ffn=4096), replace(SMALL_SMOL, layers=2, ffn=8224)],
+    ids=["q8_0", "q5_k", "q2_k", "q8_0_tall"])
+def test_a_client_in_any_company(ctx, form):
+    """A session's step takes one form of each matvec for two to eight clients:
+    a client's prompt and steps give the same bits whatever their number.  One client alone runs the batch-1 kernels: the
+    decoder's bar, 1e-3 of the largest logit, and the same tokens."""
+    model = Model(ctx, form)
+    model.synth(31)
+    rng = np.random.default_rng(5)
+    prompts = rng.integers(0, form.vocab, size=(8, 9)).astype(np.uint32)
+    feed = rng.integers(0, form.vocab, size=(4, 8)).astype(np.uint32)
+
+    def run(n):
+        s = Session(model, n, 32)
+        first = s.generate(prompts[:n], 1)[:, 0]
+        steps = [s.decode_step(f[:n], want_logits=True) for f in feed]
+        return first, [nxt for nxt, _ in steps], [logits for _, logits in steps]
+
+    whole = run(8)
+    for n in (2, 3, 4, 5, 7):
+        first, nxt, logits = run(n)
+        assert np.array_equal(first, whole[0][:n]), n
+        for i in range(len(feed)):
+            assert np.array_equal(logits[i], whole[2][i][:n]), (n, i)
+            assert np.array_equal(nxt[i], whole[1][i][:n]), (n, i)
+    first, nxt, logits = run(1)
+    assert first[0] == whole[0][0]
+    for i in range(len(feed)):
+        assert np.max(np.abs(logits[i][0] - whole[2][i][0])) <= 1e-3 * np.max(np.abs(whole[2][i][0]))
+        assert nxt[i][0] == whole[1][i][0]
