@@ -35,8 +35,9 @@ struct emu_ctx {
     void *pf_ws = nullptr; // prompt pass workspace (model.hip), grown on demand
     size_t pf_ws_bytes = 0;
     // Partial results of ops.hip's two-launch calls (kEmuScratchFloats), there
-    // from the context's creation on: such a call allocates nothing and may be
-    // captured.  Calls on a context follow each other on its stream.
+    // from the context's creation on, so that such a call allocates nothing.
+    // Calls on a context follow each other on its stream; a call that is being
+    // captured must not use it (the graph may be replayed beside them).
     float *scratch = nullptr;
 };
 constexpr size_t kEmuScratchFloats = (size_t)1 << 20; // 4 MiB

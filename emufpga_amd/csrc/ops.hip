@@ -529,7 +529,17 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 float *g_scratch[kMaxDevices] = {};
 
-// How a call runs, from its arguments alone (so the two entry points agree).
+// Whether the context's stream is being captured.  A graph outlives the call
+// and may be replayed beside the context's own, on another stream or after its
+// end: such a call leaves the context's scratch alone and runs in one launch.
+bool capturing(emu_ctx *ctx)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// How a call runs, from its arguments (so the two entry points agree) and
+// whether it may be split over chunks that meet in scratch.
 struct AttendPlan {
     bool rows;           // attend_rows_kernel, else the general form
     int chunk, chunks;   // positions per workgroup, and how many
@@ -539,7 +549,7 @@ struct AttendPlan {
 };
 
 AttendPlan attend_plan(const float *q, const void *k, const void *v, int kv_f16, int positions, int heads, int kv_heads,
-                       int hd)
+                       int hd, bool split)
 {
     AttendPlan p{};
     const int per = kv_f16 ? 8 : 4; // values per 16-byte piece
@@ -564,7 +574,7 @@ AttendPlan attend_plan(const float *q, const void *k, const void *v, int kv_f16,
     // against 10.2 in two launches; 9 on 3 of 64: 5.2, 6.3 and 8.5 against 8.7).
     int most = std::min(kAttendMaxChunks, std::max(1, 1024 / (kv_heads * p.nhg)));
     most = (int)std::min<size_t>((size_t)most, kAttendScratchFloats / ((size_t)heads * (hd + 2)));
-    most = positions <= 3 * kAttendBlock ? 1 : std::max(1, most);
+    most = positions <= 3 * kAttendBlock || !split ? 1 : std::max(1, most);
     const int blocks = (positions + kAttendBlock - 1) / kAttendBlock;
     p.chunk = (blocks + most - 1) / most * kAttendBlock;
     p.chunks = (positions + p.chunk - 1) / p.chunk;
@@ -643,7 +653,8 @@ extern "C" int emu_attend_cached(emu_ctx *ctx, const float *d_q, const void *d_k
     if (!ctx || !d_q || !d_keys || !d_values || !d_out || head_dim == 0) return EMU_E_ARG;
     if (kv_heads == 0 || heads % kv_heads != 0) return EMU_E_CONFIG; // attend.rs:82-85
     if (positions == 0 || heads == 0) return EMU_OK;
-    const AttendPlan p = attend_plan(d_q, d_keys, d_values, kv_f16, (int)positions, (int)heads, (int)kv_heads, (int)head_dim);
+    const AttendPlan p = attend_plan(d_q, d_keys, d_values, kv_f16, (int)positions, (int)heads, (int)kv_heads,
+                                     (int)head_dim, !capturing(ctx));
     AttendCall c{d_q, d_keys, d_values, (int)positions, (int)heads, (int)kv_heads, (int)head_dim, scale, nullptr, d_out};
     if (p.rows) { // at most kAttendScratchFloats
         c.ws = ctx->scratch;
@@ -673,7 +684,8 @@ extern "C" int emu_attend_cached_noalloc(emu_ctx *ctx, const float *d_q, const v
     }
     float *ws = ctx->device >= 0 && ctx->device < kMaxDevices ? g_scratch[ctx->device] : nullptr;
     if (!ws) return EMU_E_ARG; // no context set this device up
-    const AttendPlan p = attend_plan(d_q, d_keys, d_values, kv_f16, (int)positions, (int)heads, (int)kv_heads, (int)head_dim);
+    const AttendPlan p = attend_plan(d_q, d_keys, d_values, kv_f16, (int)positions, (int)heads, (int)kv_heads,
+                                     (int)head_dim, true);
     const AttendCall c{d_q, d_keys, d_values, (int)positions, (int)heads, (int)kv_heads, (int)head_dim, scale, ws, d_out};
     return attend(ctx, p, c, kv_f16);
 }
@@ -700,10 +712,11 @@ extern "C" int emu_argmax(emu_ctx *ctx, const float *d_x, uint32_t n_rows, uint3
     // workgroup and scalar loads a row, 4.8 + 1.8 so; one of 262144: 39, 4.5 +
     // 1.5).  Below 32768 or beyond 32 rows the second launch costs what the
     // chunks save: 65 rows of 151936 take 21.7 us whole (54 with scalar
-    // loads), 64 in chunks 18.6 + 3.9.  The keys go to the context's scratch.
+    // loads), 64 in chunks 18.6 + 3.9.  The keys go to the context's scratch;
+    // a captured call takes whole rows.
     const uint32_t rows = std::min(n_rows, 65535u); // a grid's second dimension; the rest in further launches
     int chunks = 1;
-    if (n_rows <= 32 && width >= 32768) chunks = (int)std::min(64u, (width + 4095) / 4096);
+    if (n_rows <= 32 && width >= 32768 && !capturing(ctx)) chunks = (int)std::min(64u, (width + 4095) / 4096);
     const int chunk = (int)((((size_t)width + chunks - 1) / chunks + 3) / 4 * 4);
     chunks = (int)(((size_t)width + chunk - 1) / chunk);
     uint64_t *keys = chunks > 1 ? reinterpret_cast<uint64_t *>(ctx->scratch) : nullptr;

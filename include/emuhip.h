@@ -252,15 +252,20 @@ int emu_rope(emu_ctx *ctx, float *d_x, uint32_t n_tok, uint32_t heads, uint32_t 
 
 /* attend_cached (spm-kv/src/attend.rs:75-94) for one token over a cached
  * prefix of `positions` rows.  keys/values: f32 or f16 (kv_f16 != 0) rows of
- * kv_heads*head_dim; score = dot * scale; softmax; weighted sum of values. */
+ * kv_heads*head_dim; score = dot * scale; softmax; weighted sum of values.
+ * Prefixes of more than 192 positions are cut into chunks that meet in the
+ * context's scratch; while the stream is being captured the call runs as one
+ * launch without it (the order of the sums is another one, the time that of a
+ * single workgroup per head group), so the graph may be replayed on any stream. */
 int emu_attend_cached(emu_ctx *ctx, const float *d_q, const void *d_keys, const void *d_values,
                       int kv_f16, uint32_t positions, uint32_t heads, uint32_t kv_heads,
                       uint32_t head_dim, float scale, float *d_out);
 /* emu_attend_cached that allocates nothing.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under HIP graph
- * capture, tight serving loops, harnesses that forbid hipMalloc).  The scores
- * go to a fixed device scratch of 1,048,576 floats (4 MiB) per device, held
- * until the process ends: heads * positions beyond that is EMU_E_CONFIG.
+ * capture, tight serving loops, harnesses that forbid hipMalloc).  The chunks'
+ * partial results (or the scores, where rows are not whole aligned 16-byte
+ * pieces) go to a fixed device scratch of 1,048,576 floats (4 MiB) per device,
+ * held until the process ends: heads * positions beyond that is EMU_E_CONFIG.
  * Calls that overlap on one device share that scratch and race. */
 int emu_attend_cached_noalloc(emu_ctx *ctx, const float *d_q, const void *d_keys, const void *d_values,
                               int kv_f16, uint32_t positions, uint32_t heads, uint32_t kv_heads,
@@ -363,7 +368,9 @@ int emu_expert_cache_policy_trace(uint32_t n_slots, int layer_aware, const uint3
 
 /* Greedy selection over n_rows rows of width: tie_last 0 = lowest index of the
  * maximum (top_k, spm-qwen3-slice/src/math.rs:38-48); 1 = last index
- * (max_by(partial_cmp), spm-batch/tests/batching.rs:111-123). */
+ * (max_by(partial_cmp), spm-batch/tests/batching.rs:111-123).  Up to 32 rows
+ * of 32768 or more are cut into chunks that meet in the context's scratch, but
+ * not while the stream is being captured: a graph holds one launch and no state. */
 int emu_argmax(emu_ctx *ctx, const float *d_x, uint32_t n_rows, uint32_t width, int tie_last,
                int32_t *d_out);
 

@@ -71,3 +71,80 @@ def test_argmax_forms(ctx, rows, width, shift):
         for r in check:
             if not (tie_last and np.isnan(x[r]).any()):
                 assert got[r] == oracle.argmax(x[r], tie_last), (r, tie_last)
+
+
+class Capture:
+    """What the context's stream is given inside `with` goes into a graph."""
+
+    def __init__(self, ctx):
+        self.hip, self.stream = C.CDLL(ctx.lib._name), C.c_void_p()  # the HIP runtime it is linked to
+        ctx.check(ctx.lib.emu_ctx_stream(ctx.h, C.byref(self.stream)), "stream")
+        self.graph, self.exec = C.c_void_p(), C.c_void_p()
+
+    def call(self, name, *args):
+        assert getattr(self.hip, name)(*args) == 0, name
+
+    def __enter__(self):
+        self.call("hipStreamBeginCapture", self.stream, C.c_int(2))  # relaxed
+        return self
+
+    def __exit__(self, *exc):
+        self.call("hipStreamEndCapture", self.stream, C.byref(self.graph))
+        if exc[0] is None:
+            self.call("hipGraphInstantiate", C.byref(self.exec), self.graph, None, None, C.c_size_t(0))
+
+    def nodes(self):
+        n = C.c_size_t()
+        self.call("hipGraphGetNodes", self.graph, None, C.byref(n))
+        return n.value
+
+    def replay(self, stream):
+        self.call("hipGraphLaunch", self.exec, stream)
+        self.call("hipStreamSynchronize", stream)
+
+
+def test_captured_calls_hold_no_scratch_of_the_context(ctx):
+    """A graph with an argmax over long rows and an attention over a long prefix
+    is one launch each, replayed on a stream of its own between the context's
+    eager calls of the same kinds, and once more when its context is gone."""
+    from emufpga_amd.device import Context
+
+    own = Context(0)
+    rng = np.random.default_rng(8)
+    rows, width, heads, hd, positions = 4, 100_001, 8, 64, 1000
+    x = rng.normal(size=(rows, width)).astype(np.float32)
+    q = rng.normal(size=heads * hd).astype(np.float32)
+    kv = rng.normal(size=(2, positions, 2 * hd)).astype(np.float16)
+    bx, bq, bk, bv = (ctx.upload(a) for a in (x, q, kv[0], kv[1]))
+    bi, bo, be, bf = ctx.alloc(4 * rows), ctx.alloc(4 * q.size), ctx.alloc(4 * rows), ctx.alloc(4 * q.size)
+
+    def calls(c, i, o):
+        c.check(c.lib.emu_argmax(c.h, bx.ptr, rows, width, 0, i.ptr), "argmax")
+        c.check(c.lib.emu_attend_cached(c.h, bq.ptr, bk.ptr, bv.ptr, 1, positions, heads, 2, hd, 0.125, o.ptr), "attend")
+
+    with Capture(own) as g:
+        calls(own, bi, bo)
+    assert g.nodes() == 2
+    beside = C.c_void_p()
+    g.call("hipStreamCreate", C.byref(beside))
+    k, v = (np.repeat(a.reshape(positions, 2, hd).astype(np.float64), heads // 2, axis=1) for a in kv)
+    p = np.exp(np.einsum("phd,hd->ph", k, q.reshape(heads, hd)) * 0.125)
+    want = np.einsum("ph,phd->hd", p / p.sum(0), v)
+    for last in (False, False, True):
+        bi.zero()
+        bo.zero()
+        ctx.sync()
+        if last:
+            own.close()
+        else:
+            calls(own, be, bf)  # the context's own, beside the replay
+        g.replay(beside)
+        if not last:
+            own.sync()
+            assert np.array_equal(be.read(np.int32), np.argmax(x, axis=1))
+            assert np.allclose(bf.read(np.float32), want.reshape(-1), rtol=2e-5, atol=2e-6)
+        assert np.array_equal(bi.read(np.int32), np.argmax(x, axis=1))
+        assert np.allclose(bo.read(np.float32), want.reshape(-1), rtol=2e-5, atol=2e-6)
+    g.call("hipGraphExecDestroy", g.exec)
+    g.call("hipGraphDestroy", g.graph)
+    g.call("hipStreamDestroy", beside)
