@@ -365,48 +365,40 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t k)
     return k;
 }
 
-// The greatest key of elements begin .. end - 1 of a row, by a workgroup of
-// 1024 (every thread gets it): float4s where the row is aligned, eight of
-// them in flight.
-__device__ __forceinline__ uint64_t row_max_key(const float *xr, int begin, int end, int tie_last, uint64_t *red)
+// One workgroup per (chunk of a row, row); with one chunk per row its index,
+// else the chunk's key for argmax_pick_kernel.  float4s from the chunk's first
+// aligned element on, four of them in flight.
+__global__ __launch_bounds__(1024) void argmax_kernel(const float *x, int width, int chunk, int tie_last, uint64_t *keys,
+                                                      int32_t *out)
 {
+    __shared__ uint64_t red[16];
+    const int begin = blockIdx.x * chunk, end = min(width, begin + chunk), tid = threadIdx.x;
+    const float *xr = x + (size_t)blockIdx.y * width;
     uint64_t best = 0;
     auto take = [&](float v, int i) {
         const uint64_t k = select_key(v, (uint32_t)i, tie_last);
         best = k > best ? k : best;
     };
-    if (reinterpret_cast<uintptr_t>(xr) % 16 == 0 && begin % 4 == 0) {
-        const int whole = end / 4 * 4;
+    const int lead = min((int)(-(reinterpret_cast<uintptr_t>(xr + begin) / 4) & 3), end - begin);
+    const int first = begin + lead, whole = first + (end - first) / 4 * 4;
+    if (tid < lead) take(xr[begin + tid], begin + tid);
 #pragma unroll 4
-        for (int i = begin + 4 * threadIdx.x; i < whole; i += 4 * blockDim.x) {
-            const float4 v = *reinterpret_cast<const float4 *>(xr + i);
-            take(v.x, i);
-            take(v.y, i + 1);
-            take(v.z, i + 2);
-            take(v.w, i + 3);
-        }
-        if (whole + (int)threadIdx.x < end && whole >= begin) take(xr[whole + threadIdx.x], whole + threadIdx.x);
-    } else {
-#pragma unroll 4
-        for (int i = begin + threadIdx.x; i < end; i += blockDim.x) take(xr[i], i);
+    for (int i = first + 4 * tid; i < whole; i += 4 * blockDim.x) {
+        const float4 v = *reinterpret_cast<const float4 *>(xr + i);
+        take(v.x, i);
+        take(v.y, i + 1);
+        take(v.z, i + 2);
+        take(v.w, i + 3);
     }
+    if (whole + tid < end) take(xr[whole + tid], whole + tid);
     best = wave_max_u64(best);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
-    __syncthreads();
-    best = red[0];
-    for (int i = 1; i < (int)(blockDim.x >> 6); ++i) best = red[i] > best ? red[i] : best;
-    return best;
-}
-
-// One workgroup per (chunk of a row, row); with one chunk per row its index,
-// else the chunk's key for argmax_pick_kernel.
-__global__ __launch_bounds__(1024) void argmax_kernel(const float *x, int width, int chunk, int tie_last, uint64_t *keys,
-                                                      int32_t *out)
-{
-    __shared__ uint64_t red[16];
-    const int begin = blockIdx.x * chunk, end = min(width, begin + chunk);
-    const uint64_t best = row_max_key(x + (size_t)blockIdx.y * width, begin, end, tie_last, red);
-    if (threadIdx.x != 0) return;
+    if (blockDim.x > EMU_WAVE) { // uniform
+        if ((tid & 63) == 0) red[tid >> 6] = best;
+        __syncthreads();
+        if (tid >= EMU_WAVE) return;
+        best = wave_max_u64(tid < (int)(blockDim.x >> 6) ? red[tid] : 0);
+    }
+    if (tid != 0) return;
     if (keys) keys[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = best;
     else out[blockIdx.y] = (int32_t)key_index(best, tie_last);
 }
@@ -708,21 +700,24 @@ extern "C" int emu_argmax(emu_ctx *ctx, const float *d_x, uint32_t n_rows, uint3
     if (!ctx || !d_x || !d_out || width == 0) return EMU_E_ARG;
     if (n_rows == 0) return EMU_OK;
     // Long rows, where few, are cut into up to 64 chunks of 4096 or more, whose
-    // keys a second launch picks from (4 rows of 151936: 24.9 us with one
-    // workgroup and scalar loads a row, 4.8 + 1.8 so; one of 262144: 39, 4.5 +
-    // 1.5).  Below 32768 or beyond 32 rows the second launch costs what the
-    // chunks save: 65 rows of 151936 take 21.7 us whole (54 with scalar
-    // loads), 64 in chunks 18.6 + 3.9.  The keys go to the context's scratch;
-    // a captured call takes whole rows.
+    // keys a second launch picks from (4 rows of 151936: 24.8 us with one
+    // workgroup and scalar loads a row, 6.4 so; one of 262144: 38.3, 6.4).  Up to
+    // 49152 a row takes no longer whole than the two launches (32767: 4.9
+    // against 6.5), beyond 32 rows the second launch costs what the chunks save
+    // (33 rows of 49155: 6.4 whole).  The keys go to the context's scratch; a
+    // captured call takes whole rows.
     const uint32_t rows = std::min(n_rows, 65535u); // a grid's second dimension; the rest in further launches
     int chunks = 1;
-    if (n_rows <= 32 && width >= 32768 && !capturing(ctx)) chunks = (int)std::min(64u, (width + 4095) / 4096);
+    if (n_rows <= 32 && width > 49152 && !capturing(ctx)) chunks = (int)std::min(64u, (width + 4095) / 4096);
     const int chunk = (int)((((size_t)width + chunks - 1) / chunks + 3) / 4 * 4);
     chunks = (int)(((size_t)width + chunk - 1) / chunk);
     uint64_t *keys = chunks > 1 ? reinterpret_cast<uint64_t *>(ctx->scratch) : nullptr;
+    // Four float4s per thread (1000 rows of 1000 took 9.1 us at 1024 threads
+    // whatever the width, 3.7 so).
+    const unsigned threads = (unsigned)std::min(1024, std::max(1, (chunk + 1023) / 1024) * EMU_WAVE);
     for (uint32_t r = 0; r < n_rows; r += rows) {
         const uint32_t n = std::min(rows, n_rows - r);
-        hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)chunks, n), dim3(1024), 0, ctx->stream, d_x + (size_t)r * width,
+        hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)chunks, n), dim3(threads), 0, ctx->stream, d_x + (size_t)r * width,
                            (int)width, chunk, tie_last ? 1 : 0, keys, d_out + r);
         EMU_LAUNCH_CHECK(ctx);
     }

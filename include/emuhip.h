@@ -369,7 +369,7 @@ int emu_expert_cache_policy_trace(uint32_t n_slots, int layer_aware, const uint3
 /* Greedy selection over n_rows rows of width: tie_last 0 = lowest index of the
  * maximum (top_k, spm-qwen3-slice/src/math.rs:38-48); 1 = last index
  * (max_by(partial_cmp), spm-batch/tests/batching.rs:111-123).  Up to 32 rows
- * of 32768 or more are cut into chunks that meet in the context's scratch, but
+ * of more than 49152 are cut into chunks that meet in the context's scratch, but
  * not while the stream is being captured: a graph holds one launch and no state. */
 int emu_argmax(emu_ctx *ctx, const float *d_x, uint32_t n_rows, uint32_t width, int tie_last,
                int32_t *d_out);

@@ -49,9 +49,10 @@ def test_rms_norm_in_place(ctx):
     assert np.allclose(bx.read(np.float32).reshape(5, 1028), exact, rtol=4e-6, atol=0)
 
 
-@pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("rows,width", [(1, 1), (3, 3), (2, 1023), (2, 32767), (2, 32768), (3, 32769), (1, 49155),
-                                        (32, 32769), (33, 32769), (1, 262144), (2, 262147), (70000, 5)])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+@pytest.mark.parametrize("rows,width", [(1, 1), (3, 3), (2, 1023), (3, 1025), (2, 32767), (2, 32768), (3, 32769), (2, 49152),
+                                        (1, 49155), (32, 32769), (33, 32769), (32, 49153), (33, 49153), (1, 262144),
+                                        (2, 262147), (70000, 5)])
 def test_argmax_forms(ctx, rows, width, shift):
     """Ties at the ends of rows and chunks under both rules, signed zeros,
     infinities, NaN (under the total order, which only the first-index rule
