@@ -15,6 +15,8 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kThreads = 256;
@@ -443,14 +445,21 @@ int launch_fmt(emu_ctx *ctx, const QmvArgs &a, int n_tok, int *key_slots)
 // HBM bound.  Each lane decodes one unit, whose eight-value groups lie apart
 // from its neighbours'; stored from there, every instruction wrote halves of
 // lines.  A wavefront's units are one contiguous run of the output: they go
-// through its own LDS and out as 1 KB non-temporal stores (nothing of a large
-// result is still in a cache when it is read).  12288 x 4096, us before ->
-// through LDS -> and non-temporal: Q6_K 55.3 -> 43.8 -> 33.7 (7.2 TB/s), Q8_0
-// 71.0 -> 46.3 -> 35.5, Q5_K 76.8 -> 41.0 -> 33.5, Q2_K 41.8 -> 39.6 -> 33.9;
-// 1024 x 4096: Q8_0 and Q5_K 6.2 -> 4.1, the others 4.2 -> 4.1.
+// through its own LDS and out as 1 KB stores, non-temporal (NT) for a large
+// result.  12288 x 4096, us with each lane's own stores -> through LDS -> and
+// non-temporal, over outputs that are not cached: Q6_K 54.2 -> 43.9 -> 40.1,
+// Q8_0 73.4 -> 44.8 -> 43.3, Q5_K 74.3 -> 40.9 -> 38.6, Q2_K 41.9 -> 41.1 ->
+// 36.0 (one output again and again: Q6_K 55.3 -> 43.8 -> 33.7).
+// What is stored so has left the caches when it is read.  The decode and a
+// reader of its result, us as above: 1024 x 4096 (16 MB) Q6_K 15.1 -> 14.5 ->
+// 16.6, Q8_0 17.6 -> 14.3 -> 16.5; 4096 x 4096 (64 MB) Q6_K 35.6 -> 32.8 ->
+// 31.3; 12288 x 4096 (192 MB) Q6_K 82.9 -> 73.0 -> 80.4, Q2_K 73.7 -> 73.7 ->
+// 78.9; 24576 x 4096 (384 MB) Q6_K 195 -> 173 -> 148.  So above 32 MB, where the
+// pair is the faster for it than with each lane's own stores; Q2_K, which gains
+// least, above the 256 MB that the Infinity Cache holds.
 // The 16-byte slots' low bits take bits 4 and 5, so that eight lanes' writes
 // meet every bank once in all four formats.
-template <class F>
+template <class F, bool NT>
 __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t *src, size_t nblocks,
                                                            float *out)
 {
@@ -486,7 +495,10 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t *src, s
     for (int i = 0; i < S; ++i) {
         const int idx = lane + EMU_WAVE * i;
         const f4 v = mine[at(idx)];
-        if ((size_t)idx < left) __builtin_nontemporal_store(v, dst + idx);
+        if ((size_t)idx < left) {
+            if constexpr (NT) __builtin_nontemporal_store(v, dst + idx);
+            else dst[idx] = v;
+        }
     }
 }
 
@@ -496,8 +508,11 @@ int launch_dequant(emu_ctx *ctx, const uint8_t *src, size_t nblocks, float *out)
     const size_t units = nblocks * F::UPB;
     if (units == 0) return EMU_OK;
     const size_t blocks = (units + kThreads - 1) / kThreads;
-    hipLaunchKernelGGL(dequant_kernel<F>, dim3((unsigned)blocks), dim3(kThreads), 0, ctx->stream, src,
-                       nblocks, out);
+    const size_t cached = (size_t)(std::is_same<F, FmtQ2K>::value ? 256 : 32) << 20; // see dequant_kernel
+    if (nblocks * F::BE * sizeof(float) > cached)
+        hipLaunchKernelGGL((dequant_kernel<F, true>), dim3((unsigned)blocks), dim3(kThreads), 0, ctx->stream, src, nblocks, out);
+    else
+        hipLaunchKernelGGL((dequant_kernel<F, false>), dim3((unsigned)blocks), dim3(kThreads), 0, ctx->stream, src, nblocks, out);
     EMU_LAUNCH_CHECK(ctx);
     return EMU_OK;
 }
