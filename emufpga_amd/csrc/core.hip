@@ -90,7 +90,6 @@ extern "C" int emu_ctx_destroy(emu_ctx *ctx)
     for (auto &ev : ctx->events)
         if (ev) (void)hipEventDestroy(ev);
     if (ctx->mfma_ws) (void)hipFree(ctx->mfma_ws);
-    if (ctx->pf_ws) (void)hipFree(ctx->pf_ws);
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     for (int i = 0; i < 2; ++i) {
         if (ctx->stage_ev[i]) (void)hipEventDestroy(ctx->stage_ev[i]);

@@ -32,8 +32,6 @@ struct emu_ctx {
     void *stage[2] = {};         // pinned host staging for file -> HBM uploads (files.hip)
     hipEvent_t stage_ev[2] = {}; // the copy out of each staging buffer
     size_t stage_bytes = 0;
-    void *pf_ws = nullptr; // prompt pass workspace (model.hip), grown on demand
-    size_t pf_ws_bytes = 0;
     // Partial results of ops.hip's two-launch calls (kEmuScratchFloats), there
     // from the context's creation on, so that such a call allocates nothing.
     // Calls on a context follow each other on its stream; a call that is being

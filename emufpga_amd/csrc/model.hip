@@ -103,6 +103,10 @@ struct emu_model {
     bool prs_dirty = true;
     size_t prs_qkv = 0, prs_o = 0, prs_g = 0, prs_u = 0, prs_d = 0, prs_r = 0, prs_ge = 0, prs_ue = 0, prs_de = 0,
            prs_layer = 0;
+    // The prompt pass's workspace, grown on demand: its sessions run on the
+    // context's stream one after another and share it.
+    void *pf_ws = nullptr;
+    size_t pf_ws_bytes = 0;
     void touched() { lm_dirty = prs_dirty = true; } // the weights may have changed
 };
 
@@ -1642,18 +1646,19 @@ PromptBufs prompt_bufs(const emu_model *m, int N, const PromptSplits &ks, uint8_
     return b;
 }
 
-int prompt_reserve(emu_ctx *ctx, size_t bytes)
+int prompt_reserve(emu_model *m, size_t bytes)
 {
-    if (bytes <= ctx->pf_ws_bytes) return EMU_OK;
-    if (ctx->pf_ws) {
-        EMU_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        EMU_HIP(ctx, hipFree(ctx->pf_ws));
-        ctx->pf_ws = nullptr;
-        ctx->pf_ws_bytes = 0;
+    if (bytes <= m->pf_ws_bytes) return EMU_OK;
+    if (m->pf_ws) {
+        EMU_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
+        emu_free(m->ctx, m->pf_ws);
+        m->pf_ws = nullptr;
+        m->pf_ws_bytes = 0;
     }
-    EMU_HIP(ctx, hipMalloc(&ctx->pf_ws, bytes));
-    ctx->pf_ws_bytes = bytes;
-    return EMU_OK;
+    const int st = emu_malloc(m->ctx, bytes, &m->pf_ws);
+    if (st == EMU_OK) m->pf_ws_bytes = bytes;
+    else m->pf_ws = nullptr;
+    return st;
 }
 
 // Tokens t0 .. t0 + tc - 1 of every client's prompt: the layers' keys and
@@ -1857,7 +1862,7 @@ int run_prompt(emu_session *s, uint32_t prompt_len, uint32_t *done)
     ks.d = F ? emu_pf_split(H, 1, F, count) : 1;
     ks.r = m->moe() ? emu_pf_split((int)c.n_experts, 1, H, count) : 1;
     const size_t bytes = prompt_bufs(m, (int)s->n * tc_max, ks, nullptr).bytes;
-    int st = prompt_reserve(m->ctx, bytes);
+    int st = prompt_reserve(m, bytes);
     if (st == EMU_OK) st = prompt_scales(m);
     if (st == EMU_E_NOMEM) { // one token per step, as ever
         (void)hipGetLastError();
@@ -1866,7 +1871,7 @@ int run_prompt(emu_session *s, uint32_t prompt_len, uint32_t *done)
     if (st != EMU_OK) return st;
     for (int t0 = 0; t0 < count; t0 += tc_max) {
         const int tc = std::min(tc_max, count - t0);
-        const PromptBufs b = prompt_bufs(m, (int)s->n * tc, ks, static_cast<uint8_t *>(m->ctx->pf_ws));
+        const PromptBufs b = prompt_bufs(m, (int)s->n * tc, ks, static_cast<uint8_t *>(m->pf_ws));
         if ((st = prompt_chunk(s, b, ks, t0, tc)) != EMU_OK) return st;
         for (auto &p : s->host_pos) p += (uint32_t)tc;
         *done += (uint32_t)tc;
@@ -2049,6 +2054,7 @@ extern "C" int emu_model_destroy(emu_model *m)
     if (m->lm) emu_free(m->ctx, m->lm);
     if (m->mm) emu_free(m->ctx, m->mm);
     if (m->prs) emu_free(m->ctx, m->prs);
+    if (m->pf_ws) emu_free(m->ctx, m->pf_ws);
     delete m;
     return EMU_OK;
 }

@@ -489,8 +489,8 @@ int emu_decode_step(emu_session *s, const uint32_t *h_tokens, uint32_t *h_next, 
  * positions and step counts that the steps leave.  Prompts go one token per
  * step with EMU_SESSION_F32_ACT, an attached expert cache, Zipf
  * routing or a route trace (defined per step), rows of more than 16384
- * columns, or no device memory for the pass's workspace (kept by the context,
- * for at most 2048 tokens at a time). */
+ * columns, or no device memory for the pass's workspace (kept by the model
+ * until it is destroyed, for at most 2048 tokens at a time). */
 int emu_generate(emu_session *s, const uint32_t *h_prompt, uint32_t prompt_len, uint32_t steps,
                  uint32_t *h_out);
 /* Time `steps` greedy steps (after the caller's warmup) with events around the

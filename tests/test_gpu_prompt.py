@@ -8,6 +8,7 @@ norm for the cache, the decoder's 1e-3 of the largest logit for the logits.
 Prompt lengths sit at the edges of the pass's tiles (32, 64, 128 tokens) and
 of its range (4 tokens; more than 2048 over all clients take several passes).
 """
+import ctypes as C
 from dataclasses import replace
 
 import numpy as np
@@ -258,3 +259,31 @@ def test_cache_entries_that_overflow_f16(ctx, form, what):
                     after += int(np.sum(fine[first:]))
         assert first > 0 and (c or first < plen)
     assert (after > 0) == (what == "keys")
+
+
+def test_the_workspace_goes_with_the_model(ctx):
+    """A long prompt's workspace (about 100 MB here) is held while the model lives,
+    not until the context ends."""
+    free, total = C.c_size_t(), C.c_size_t()
+    hip = C.CDLL(ctx.lib._name)  # the HIP runtime it is linked to
+
+    def left():
+        ctx.sync()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    def run(plen):
+        model = Model(ctx, replace(SMALL_SMOL, layers=1))
+        model.synth(5)
+        sess = Session(model, 8, 264)
+        sess.generate(np.ones((8, plen), np.uint32), 1)
+        held = left()
+        sess.close()
+        model.close()
+        return held
+
+    run(4)  # whatever the runtime keeps from a first run
+    before = left()
+    held = run(257)
+    assert before - held > 64 << 20
+    assert left() >= before - (16 << 20)
