@@ -2313,6 +2313,7 @@ extern "C" int emu_model_resident_bytes(const emu_model *m, uint64_t *bytes)
 {
     if (!m || !bytes) return EMU_E_ARG;
     *bytes = (uint64_t)m->total + m->lm_bytes + m->mm_bytes;
+    if (m->prs) *bytes += sizeof(float) * m->prs_layer * m->cfg.layers;
     return EMU_OK;
 }
 

@@ -444,10 +444,11 @@ int emu_model_tensor(emu_model *model, int kind, uint32_t layer, void **d_ptr, s
 int emu_model_synth(emu_model *model, uint64_t seed);
 /* Rebuild what the model derives from its weights: the lane-major copy of the
  * Q6_K matrices that the batch-1 step reads (emu_weights_lane_major), the
- * matrix-core operand copy, and (at the next prompt) the prompt pass's scale
- * of every weight row.  The decode entry points do this by themselves after emu_model_synth, the GGUF loaders and any
- * emu_model_tensor call; call it after writing weights through a pointer
- * that emu_model_tensor returned earlier. */
+ * matrix-core operand copy, and, for every encoding and at the next prompt, the
+ * prompt pass's scale of every weight row.  The decode entry points do this by
+ * themselves after emu_model_synth, the GGUF loaders and any emu_model_tensor
+ * call; call it after writing weights through a pointer that emu_model_tensor
+ * returned earlier. */
 int emu_model_sync(emu_model *model);
 /* Device address of the lane-major copy: a layer (same offsets as its
  * EMU_T_LAYER tensor; only the matrices whose columns the batch-1 limb
@@ -460,7 +461,9 @@ int emu_model_weight_bytes(const emu_model *model, uint64_t *bytes);
 /* HBM the model's parameters hold: its allocation in GGUF order (every
  * tensor, norms included) plus the lane-major and matrix-core operand copies
  * of its Q6_K matrices (about three times the weights for a dense Q6_K
- * model).  No reference counterpart. */
+ * model) and, from the first prompt pass on, its scale of every weight row.
+ * The pass's workspace, which holds no parameters, is not counted.  No
+ * reference counterpart. */
 int emu_model_resident_bytes(const emu_model *model, uint64_t *bytes);
 
 /* A set of clients (spm-batch/src/session.rs:13-38 Client, :46-79 Scratch):

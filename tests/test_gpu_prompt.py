@@ -287,3 +287,19 @@ def test_the_workspace_goes_with_the_model(ctx):
     held = run(257)
     assert before - held > 64 << 20
     assert left() >= before - (16 << 20)
+
+
+@pytest.mark.parametrize("form", ["q8_0_smol", "granite", "gemma_window"])
+def test_resident_bytes_count_the_row_scales(ctx, form):
+    cfg = FORMS[form]
+    model = Model(ctx, cfg)
+    model.synth(5)
+    sess = Session(model, 1, 16)
+    sess.decode_step([1])
+    before = model.resident_bytes()
+    sess.generate(np.ones((1, 8), np.uint32), 1)
+    rows = cfg.q_width + 2 * cfg.kv_width + cfg.hidden
+    ff = cfg.shared_ff if cfg.n_experts else cfg.ffn
+    rows += (2 * ff + cfg.hidden) if ff else 0
+    rows += cfg.n_experts * (1 + 2 * cfg.expert_ff + cfg.hidden)
+    assert model.resident_bytes() - before == 4 * rows * cfg.layers
