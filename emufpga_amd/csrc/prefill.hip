@@ -6,15 +6,17 @@
 // (the last one is an ordinary decode step, which makes the logits); the KV
 // cache, positions and step counts end up as the steps would leave them.
 //
-// Arithmetic: 32-bit values on the f16 matrix cores without giving up their
-// precision.  A value v scaled by a power of two into f16's range is held as
-// hi + lo, hi = f16(v), lo = f16(v - hi), both rounded to nearest: exact to
-// 2^-24 of |v| (24 bits), as f32 is.  A product is hi*hi + lo*hi + hi*lo,
-// accumulated in f32 by the matrix cores; the dropped lo*lo is below 2^-24 of
-// it.  Activations carry one power of two per row, weights one per matrix row
-// (pf_rowscale_kernel).  K and V are f16 in the cache, so the attention
-// splits only the queries and the softmax weights (an f32 cache is attended
-// in f32).
+// Arithmetic: 32-bit values on the f16 matrix cores as pairs of halves
+// (split.hpp, which says what a pair holds: 23 bits, down to a floor of 2^-39
+// of the row's largest value).  A product is hi*hi + lo*hi + hi*lo, accumulated
+// in f32 by the matrix cores; lo*lo, at most 2^-22 of it, is dropped.
+// Activations carry one power of two per row, weights one per matrix row
+// (pf_rowscale_kernel).  K and V are f16 in the cache, so the attention splits
+// only the queries and the softmax weights (an f32 cache is attended in f32).
+// Against 64 bits the sums are as far off as the steps' f32 sums, within half
+// as much again (figures at pf_tile), and less than the steps' limbs from 2048
+// columns on.  What that leaves a whole turn with: a cache entry now and then
+// rounds to the neighbouring half, and the logits move by 1e-4 to 2e-4.
 //
 // No result depends on which other tokens share the launch: a row's sums run
 // over the columns in an order fixed by the weights' shape and the prompt's
@@ -355,10 +357,11 @@ __global__ __launch_bounds__(kThreads) void pf_rowscale_kernel(const uint8_t *w,
 
 // ---- the product ----------------------------------------------------------
 // Tile: MT x 32 tokens by 128 weight rows, four wavefronts of 32 rows each.
-// The tokens' planes come straight into LDS, one stage of the tallest tile
-// or two of the others at a time, double buffered with one barrier each, and serve all four wavefronts; each lane decodes its own
-// row's weights in registers, in the matrix cores' operand order, so weights
-// never pass through LDS and are decoded once per MT x 32 tokens.
+// The tokens' planes come straight into LDS, one stage of the tallest tile or
+// two of the others at a time, double buffered with one barrier each, and serve
+// all four wavefronts; each lane decodes its own row's weights in registers, in
+// the matrix cores' operand order, so weights never pass through LDS and are
+// decoded once per MT x 32 tokens.
 typedef const __attribute__((address_space(1))) void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
 
@@ -366,7 +369,7 @@ typedef __attribute__((address_space(3))) void lvoid;
 // pf_tile<D, MT, L> is one tile with its first L of MT token fragments live
 // (the others hold no tokens): L is a constant in it, because a branch on the
 // live count around each matrix instruction kept them from overlapping with
-// the decode (gate|up of 4096 columns at 511 tokens: 335 us with them).
+// the decode (gate|up of 4096 columns at 511 tokens: 335 us with them, 320 so).
 template <class D, int MT, int L>
 __device__ __forceinline__ void pf_tile(const PfGemm &g, uint8_t *lds, int a0, int count, int expert, int mat, int r0)
 {
@@ -623,7 +626,8 @@ template <int G, int NS, bool MOE> __global__ __launch_bounds__(kRowThreads) voi
 
 // A gate|up pair's partial sums -> the activation -> the down product's
 // operands.  rows_used (expert rows): the padded row count, and src < 0 marks
-// padding.
+// padding.  Rows wider than 8192 in more than four shares (G 4, NS 8: prompts of
+// few tokens) spill 110 registers; such a launch waits for its partial sums.
 template <int G, int NS>
 __global__ __launch_bounds__(kRowThreads) void pf_glu_kernel(const float *part, int nks, size_t ks_stride,
                                                              size_t mat_stride, int F, int act, PfPlanes P,
@@ -773,6 +777,7 @@ __global__ __launch_bounds__(kThreads) void pf_heads_kernel(PfHeads a)
 // cores with a lane's column its query row, so the softmax state is one value
 // per lane, and the weights are already the next product's operand (its
 // position order is the one the scores' registers have; V^T is read to match).
+// 511 tokens, 32 heads on 8 of 128: 40 us per layer.
 // Queries and weights are hi + lo halves; the weights carry a factor 2^15 so
 // that small ones keep their bits.
 constexpr int kAttnPos = 64; // positions per K/V tile
@@ -872,7 +877,8 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
     const int w_first = base + min(r0 + 32 * w, rows - 1) / G; // and its first
     const int w_lo = a.window > 0 && w_last + 1 > a.window ? w_last + 1 - a.window : 0; // the last row's window
     const size_t cache = (((size_t)client * a.layers + a.layer) * a.kv_heads + kvh) * (size_t)a.context * HD;
-    const _Float16 *kc = static_cast<const _Float16 *>(a.k_cache) + cache, *vc = static_cast<const _Float16 *>(a.v_cache) + cache;
+    const _Float16 *kc = static_cast<const _Float16 *>(a.k_cache) + cache;
+    const _Float16 *vc = static_cast<const _Float16 *>(a.v_cache) + cache;
 
     half8 qh[NS], ql[kLoLds ? 1 : NS];
     {
@@ -1032,7 +1038,7 @@ __global__ __launch_bounds__(EMU_WAVE *WV, HD > 128 ? 1 : 2) void pf_attn_kernel
 // LPR lanes hold a row, four values each; a wavefront takes 16 of each 64
 // positions, each lane group with a softmax state of its own, merged in LDS
 // (the shape of attend_rows_kernel).  511 tokens over 32 heads on 8 of 128:
-// 0.23 ms per layer, bound by the L2 reads of K and V (the f16 cache's 49 us on
+// 0.23 ms per layer, bound by the L2 reads of K and V (the f16 cache's 40 us on
 // the matrix cores); fed a token per step, a prompt of 256 took 447 ms on
 // Qwen3-8B, and 19 so.
 template <int LPR, int GH>
@@ -1248,7 +1254,8 @@ int emu_pf_split(int rows, int nmat, int cols, int prompt)
     // that short matrices and short prompts still fill the chip: the count
     // with the least rounds x (stages + a start-up of about three), plus what
     // writing and reading a share's sums costs in stages.  A CU holds two
-    // workgroups of the taller tiles, four of the lowest.  Not from the number of clients: a client's sums keep their order in any company.
+    // workgroups of the taller tiles, four of the lowest.  Not from the number
+    // of clients: a client's sums keep their order in any company.
     const int spans = (cols + 255) / 256, mt = prompt <= 32 ? 1 : prompt <= 64 ? 2 : 4;
     const int tiles = nmat * ((rows + 127) / 128) * ((prompt + 32 * mt - 1) / (32 * mt));
     const int slots = 256 * (mt == 1 ? 4 : 2);
@@ -1270,12 +1277,15 @@ int emu_pf_rowscale(emu_ctx *ctx, int encoding, const uint8_t *w, size_t row_byt
     if (rows == 0) return EMU_OK;
     const dim3 grid((unsigned)((rows + 31) / 32)), block(kThreads);
     hipStream_t s = ctx->stream;
+    auto go = [&](auto enc, int nb) {
+        hipLaunchKernelGGL(pf_rowscale_kernel<decltype(enc)::value>, grid, block, 0, s, w, row_bytes, rows, nb, scale);
+    };
     switch (encoding) {
-    case EMU_ENC_Q6_K: hipLaunchKernelGGL(pf_rowscale_kernel<EMU_ENC_Q6_K>, grid, block, 0, s, w, row_bytes, rows, cols / 256, scale); break;
-    case EMU_ENC_Q5_K: hipLaunchKernelGGL(pf_rowscale_kernel<EMU_ENC_Q5_K>, grid, block, 0, s, w, row_bytes, rows, cols / 256, scale); break;
-    case EMU_ENC_Q2_K: hipLaunchKernelGGL(pf_rowscale_kernel<EMU_ENC_Q2_K>, grid, block, 0, s, w, row_bytes, rows, cols / 256, scale); break;
-    case EMU_ENC_Q8_0: hipLaunchKernelGGL(pf_rowscale_kernel<EMU_ENC_Q8_0>, grid, block, 0, s, w, row_bytes, rows, cols / 32, scale); break;
-    case EMU_ENC_F32: hipLaunchKernelGGL(pf_rowscale_kernel<EMU_ENC_F32>, grid, block, 0, s, w, row_bytes, rows, cols, scale); break;
+    case EMU_ENC_Q6_K: go(std::integral_constant<int, EMU_ENC_Q6_K>{}, cols / 256); break;
+    case EMU_ENC_Q5_K: go(std::integral_constant<int, EMU_ENC_Q5_K>{}, cols / 256); break;
+    case EMU_ENC_Q2_K: go(std::integral_constant<int, EMU_ENC_Q2_K>{}, cols / 256); break;
+    case EMU_ENC_Q8_0: go(std::integral_constant<int, EMU_ENC_Q8_0>{}, cols / 32); break;
+    case EMU_ENC_F32: go(std::integral_constant<int, EMU_ENC_F32>{}, cols); break;
     default: return EMU_E_UNSUPPORTED;
     }
     EMU_LAUNCH_CHECK(ctx);
@@ -1306,11 +1316,15 @@ int emu_pf_embed(emu_ctx *ctx, int encoding, const uint8_t *embed, size_t row_by
 {
     const dim3 grid((unsigned)(n * tc)), block(kThreads);
     hipStream_t s = ctx->stream;
+    auto go = [&](auto fmt) {
+        hipLaunchKernelGGL(pf_embed_kernel<decltype(fmt)>, grid, block, 0, s, embed, row_bytes, hidden, prompt, stride, t0,
+                           tc, h, scale);
+    };
     switch (encoding) {
-    case EMU_ENC_Q6_K: hipLaunchKernelGGL(pf_embed_kernel<FmtQ6K>, grid, block, 0, s, embed, row_bytes, hidden, prompt, stride, t0, tc, h, scale); break;
-    case EMU_ENC_Q5_K: hipLaunchKernelGGL(pf_embed_kernel<FmtQ5K>, grid, block, 0, s, embed, row_bytes, hidden, prompt, stride, t0, tc, h, scale); break;
-    case EMU_ENC_Q2_K: hipLaunchKernelGGL(pf_embed_kernel<FmtQ2K>, grid, block, 0, s, embed, row_bytes, hidden, prompt, stride, t0, tc, h, scale); break;
-    case EMU_ENC_Q8_0: hipLaunchKernelGGL(pf_embed_kernel<FmtQ8_0>, grid, block, 0, s, embed, row_bytes, hidden, prompt, stride, t0, tc, h, scale); break;
+    case EMU_ENC_Q6_K: go(FmtQ6K{}); break;
+    case EMU_ENC_Q5_K: go(FmtQ5K{}); break;
+    case EMU_ENC_Q2_K: go(FmtQ2K{}); break;
+    case EMU_ENC_Q8_0: go(FmtQ8_0{}); break;
     default: return EMU_E_UNSUPPORTED;
     }
     EMU_LAUNCH_CHECK(ctx);

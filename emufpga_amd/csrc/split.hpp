@@ -57,7 +57,8 @@ __device__ __forceinline__ half8 split8_part(const float (&x)[8], float s, float
     for (int i = 0; i < 8; i += 2) {
         const float2v p = {x[i] * s, x[i + 1] * s};
         const half2v h = __builtin_convertvector(p, half2v);
-        const float2v r = {__builtin_fmaf((float)h[0], -part, x[i] * s2), __builtin_fmaf((float)h[1], -part, x[i + 1] * s2)};
+        const float2v r = {__builtin_fmaf((float)h[0], -part, x[i] * s2),
+                           __builtin_fmaf((float)h[1], -part, x[i + 1] * s2)};
         const half2v l = __builtin_convertvector(r, half2v);
         out[i] = l[0];
         out[i + 1] = l[1];
@@ -86,8 +87,9 @@ __device__ __forceinline__ void biased8(uint32_t q0, uint32_t q1, float m, half8
 {
     const _Float16 mh = (_Float16)m, ml = (_Float16)__builtin_fmaf((float)mh, -1.0f, m);
     const half2v mh2 = {mh, mh}, ml2 = {ml, ml}, bias = {(_Float16)(-1024.0f - BIAS), (_Float16)(-1024.0f - BIAS)};
-    const uint32_t q[4] = {__builtin_amdgcn_perm(0x64646464u, q0, 0x04010400u), __builtin_amdgcn_perm(0x64646464u, q0, 0x04030402u),
-                           __builtin_amdgcn_perm(0x64646464u, q1, 0x04010400u), __builtin_amdgcn_perm(0x64646464u, q1, 0x04030402u)};
+    const uint32_t k = 0x64646464u, lo2 = 0x04010400u, hi2 = 0x04030402u;
+    const uint32_t q[4] = {__builtin_amdgcn_perm(k, q0, lo2), __builtin_amdgcn_perm(k, q0, hi2),
+                           __builtin_amdgcn_perm(k, q1, lo2), __builtin_amdgcn_perm(k, q1, hi2)};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         half2v c;
@@ -106,8 +108,9 @@ __device__ __forceinline__ void biased8(uint32_t q0, uint32_t q1, float m, half8
 template <int BIAS> __device__ __forceinline__ void codes_minus(uint32_t q0, uint32_t q1, half8 &c8)
 {
     const half2v bias = {(_Float16)(-1024.0f - BIAS), (_Float16)(-1024.0f - BIAS)};
-    const uint32_t q[4] = {__builtin_amdgcn_perm(0x64646464u, q0, 0x04010400u), __builtin_amdgcn_perm(0x64646464u, q0, 0x04030402u),
-                           __builtin_amdgcn_perm(0x64646464u, q1, 0x04010400u), __builtin_amdgcn_perm(0x64646464u, q1, 0x04030402u)};
+    const uint32_t k = 0x64646464u, lo2 = 0x04010400u, hi2 = 0x04030402u;
+    const uint32_t q[4] = {__builtin_amdgcn_perm(k, q0, lo2), __builtin_amdgcn_perm(k, q0, hi2),
+                           __builtin_amdgcn_perm(k, q1, lo2), __builtin_amdgcn_perm(k, q1, hi2)};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         half2v c;

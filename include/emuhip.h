@@ -131,7 +131,13 @@ int emu_dequant(emu_ctx *ctx, int encoding, const void *d_src, size_t src_len, f
  * columns, or at 2..8 tokens on the matrix-core widths, carries x as three
  * int8 limbs per column with a power-of-two scale per 16 columns (exact to
  * 2^-20 of each 16-column group's largest |x|) and sums codes x limbs in
- * int32.  EMU_MV_F32_ACT keeps x in f32 for every shape: each weight is
+ * int32.  A Q8_0, Q5_K or Q2_K matvec at 2..8 tokens, where its rows, columns
+ * and token count make that the faster form, carries x as two halves per column
+ * (off by at most 2^-23 of each |x|, and by 2^-51 of its 256-column span's
+ * largest) against exact integer codes, summed in f32: as close to the exact
+ * sum as f32 arithmetic (1e-7 of its norm), in another order, so a token's
+ * result may differ in the last bits with the number of tokens.
+ * EMU_MV_F32_ACT keeps x in f32 for every shape: each weight is
  * dequantized and multiplied in f32, the reference's arithmetic
  * (spm-qwen3-slice/src/math.rs:12-20) up to the order of the additions.
  * It cannot be combined with the two layout flags (EMU_E_UNSUPPORTED). */
@@ -488,8 +494,9 @@ int emu_decode_step(emu_session *s, const uint32_t *h_tokens, uint32_t *h_next, 
  * trips.  examples/serve-demo.rs:62-91 feeds one prompt token per step; here
  * a prompt of four tokens or more, but for its last token, goes through each
  * layer as one matrix product per projection (32-bit values split into pairs
- * of halves on the matrix cores, exact to 2^-24 of each), leaving the cache,
- * positions and step counts that the steps leave.  Prompts go one token per
+ * of halves on the matrix cores: off by at most 2^-23 of each, and by 2^-39 of
+ * its row's largest), leaving the cache, positions and step counts that the
+ * steps leave; a cache entry may round to the neighbouring value of its type.  Prompts go one token per
  * step with EMU_SESSION_F32_ACT, an attached expert cache, Zipf
  * routing or a route trace (defined per step), rows of more than 16384
  * columns, or no device memory for the pass's workspace (kept by the model
@@ -515,8 +522,9 @@ int emu_session_time_layers(emu_session *s, float *h_us, uint32_t n);
  *    order of the additions: spm-qwen3-slice/src/math.rs:12-20,
  *    spm-linear/src/stream.rs:31-125) instead of the int8-limb kernels
  *    (activations exact to 2^-20 of each 16- or 256-column group's largest
- *    |x|).  Slower; the mode in which greedy tokens are held identical to the
- *    reference's over long runs.
+ *    |x|), the two halves of emu_qmatvec and the prompt pass.  Slower; the
+ *    mode in which greedy tokens are held identical to the reference's over
+ *    long runs.
  *  - EMU_SESSION_DIRECT: the step's kernels are launched one by one instead
  *    of being captured once into a HIP graph and replayed (same kernels,
  *    same order, same results), for profilers and tracers.
