@@ -264,6 +264,47 @@ def test_products_of_a_row_with_one_large_value(ctx):
         assert np.linalg.norm(got[t] - want[t]) <= bar, t
 
 
+@pytest.mark.parametrize("ratio", [2.0 ** 10, 2.0 ** 20])
+@pytest.mark.parametrize("form", ["q6_k", "q5_k_no_groups", "q2_k_head256", "q8_0_smol"])
+def test_products_of_rows_with_one_large_block(ctx, form, ratio):
+    """Value rows whose first block's d is 2^10 or 2^20 times the others', over
+    activations that are zero there.  The others keep what
+    test_products_against_64_bits holds, down to 2^-25 under the power of two
+    that puts the row's bound (the block's d times the largest code) into [2^14,
+    2^15): 2^-39 of the bound in each weight, times the code (32; Q8_0 128) where
+    the block's multiplier carries it."""
+    cfg = FORMS[form]
+    be, bb = gguf.LAYOUT[cfg.encoding]
+    model = Model(ctx, cfg)
+    model.synth(12)
+    rb = gguf.row_bytes(cfg.encoding, cfg.hidden)
+    at = (cfg.q_width + cfg.kv_width) * rb
+    layer = model.read_tensor(_lib.EMU_T_LAYER, 0)
+    raw = layer[at:at + cfg.kv_width * rb]
+    per = raw.reshape(cfg.kv_width, -1, bb)
+    bound = np.zeros(cfg.kv_width)
+    largest = {_lib.Q6_K: [4096], _lib.Q5_K: [1953, 63], _lib.Q2_K: [45, 15], _lib.Q8_0: [128]}[cfg.encoding]
+    for d_at, code in zip(D_AT[cfg.encoding], largest):
+        per[:, 1:, d_at:d_at + 2] = np.array([2.0 ** -12], np.float16).view(np.uint8)
+        per[:, 0, d_at:d_at + 2] = np.array([2.0 ** -12 * ratio], np.float16).view(np.uint8)
+        bound += code * 2.0 ** -12 * ratio
+    model.write_tensor(_lib.EMU_T_LAYER, layer, 0)
+    gain = np.ones((cfg.layers, cfg.hidden), np.float32)
+    gain[0, :be] = 0.0
+    model.write_tensor(_lib.EMU_T_ATTN_NORM, gain)
+    prompts = np.random.default_rng(7).integers(0, model.cfg.vocab, size=(1, 75)).astype(np.uint32)
+    a = Session(model, 1, 77, kv_f16=False)
+    a.generate(prompts, 1)
+    w = npref.DECODERS[cfg.encoding](raw).reshape(-1, cfg.hidden).astype(np.float64)
+    embed = npref.DECODERS[cfg.encoding](model.read_tensor(_lib.EMU_T_EMBED)).reshape(-1, cfg.hidden).astype(np.float64)
+    x = embed[prompts[0, :74]]
+    x = x / np.sqrt((x * x).mean(1, keepdims=True) + cfg.eps) * gain[0]
+    want, got = x @ w.T, a.read_kv(0, 0, True, 74).astype(np.float64)
+    code = {_lib.Q6_K: 32, _lib.Q8_0: 128}.get(cfg.encoding, 1)
+    floor = 2.0 ** -39 * code * bound * np.abs(x).sum(1, keepdims=True)
+    assert np.linalg.norm(got - want) <= 1.7e-7 * np.linalg.norm(want) + np.linalg.norm(floor)
+
+
 @pytest.mark.parametrize("form", ["q5_k_no_groups", "q2_k_head256"])
 def test_queries_over_an_f32_cache_are_f32(ctx, form):
     """Two query dimensions 2^24 times the others, over keys that hold zeros
@@ -428,3 +469,24 @@ def test_resident_bytes_count_the_row_scales(ctx, form):
     rows += (2 * ff + cfg.hidden) if ff else 0
     rows += cfg.n_experts * (1 + 2 * cfg.expert_ff + cfg.hidden)
     assert model.resident_bytes() - before == 4 * rows * cfg.layers
+
+
+@pytest.mark.parametrize("kv_f16", [True, False])
+@pytest.mark.parametrize("form", ["q6_k", "q8_0_smol", "granite_deep", "olmoe_deep", "gemma_deep"])
+def test_a_prompt_in_any_company(ctx, form, kv_f16):
+    """A client's cached rows are the same bits alone (one pass of 299 tokens)
+    and among eight (two passes, of 256 and 43)."""
+    model = Model(ctx, FORMS[form])
+    model.synth(9)
+    if form.startswith("gemma"):
+        gemma_layer_scales(model)
+    prompts = np.random.default_rng(6).integers(0, model.cfg.vocab, size=(8, 300)).astype(np.uint32)
+    a, b = Session(model, 8, 304, kv_f16), Session(model, 1, 304, kv_f16)
+    a.generate(prompts, 1)
+    for c in (0, 5):
+        b.reset()
+        b.generate(prompts[c:c + 1], 1)
+        for layer in range(model.cfg.layers):
+            for values in (False, True):
+                x, y = a.read_kv(c, layer, values, 299), b.read_kv(0, layer, values, 299)
+                assert np.array_equal(x.view(np.uint32), y.view(np.uint32)), (c, layer, values)
